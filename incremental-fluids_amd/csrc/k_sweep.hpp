@@ -3,6 +3,7 @@
 // k_pcg.hip, whose kernels deal strips grouped by XCD, and by k_sweep_up.hip,
 // whose kernels deal them upstream first.
 #pragma once
+#include <cstddef>
 #include <type_traits>
 
 #include "ifl_solver.hpp"
@@ -41,40 +42,44 @@ IFL_DEV int strip_of_block(int b, int n, bool reverse, int order) {
 static int sweep_blocks(int n, int order) { return order ? n : 8 * ((n + 7) / 8); }
 
 // ---------------------------------------------------------------- streamed sweeps
-// One strip runs as a workgroup of six waves. Waves w and w + 4 of a
+// One strip runs as a workgroup of eight waves. Waves w and w + 4 of a
 // workgroup run on the same SIMD (the dispatcher deals a workgroup's waves
 // round robin over the CU's four SIMDs), and a wave issues in order, so the
-// recurrence gets a SIMD of its own and the light roles share:
+// recurrence gets a SIMD of its own and the other roles share three:
 //   wave 0        the recurrence. It only does what the dependency chain
-//                 needs: operands come from an LDS ring into registers half a
+//                 needs: operands come from an LDS ring into registers one
 //                 block ahead, FLUID masks come as 64-lane masks through scalar
 //                 loads, and results go to an LDS output ring. A single wave
 //                 issues one instruction at a time, so everything that is not
 //                 on the chain lives in the other waves;
-//   wave 1        the writer: stores the results of each finished block to
-//                 HBM, hands the edge row to the neighbouring strip, and
-//                 forms the reductions (max|r|, the z.r partial);
-//   waves 2, 3    loaders: each streams every kLoaders-th block of 8 steps
+//   wave 1        the writer: hands the edge row of each finished block to the
+//                 neighbouring strip and stores its results to HBM;
+//   waves 2, 3, 6 and 7
+//                 loaders: each streams every loaders(KIND)-th block of 8 steps
 //                 (4 KB contiguous per array in the skewed layout) from HBM
-//                 straight into the LDS ring;
+//                 through its registers into the LDS ring; the forward sweep's
+//                 also form, store and take the maximum of the new residual;
+//   wave 7        in the backward sweep the dot wave instead: the z.r partial;
 //   wave 4        idle (it would share wave 0's SIMD): returns at once;
 //   wave 5        the edge poller (sharing the writer's SIMD): fetches
 //                 upcoming inter-strip values from global memory, 64 steps
 //                 per round trip, into an LDS ring.
-// Measured at 2048^2 against eight waves (five loaders, the poller on wave
-// 1): forward sweep 551 -> 498 us, backward 541 -> 508 us.
-// Slot life cycle: loader fills -> wave 0 computes -> writer drains -> free.
-// Counters in LDS order the hand-offs (LDS instructions of one workgroup are
-// executed in order). Every wait is bounded; a timeout raises `abort`, which
-// every wave checks, so the workgroup always drains.
+// What bounds it: wave 0's steps (37 clocks each alone, the chain of four
+// FP64 operations, the select and the lane move), one CU's rate of streaming
+// memory (59-66 GB/s from HBM, 100 from the Infinity Cache, 141 from L2), and
+// the hand-offs between strips.
+// Slot life cycle: loader fills -> wave 0 computes -> writer (and dot wave)
+// drain -> free. Counters in LDS order the hand-offs (LDS instructions of one
+// workgroup are executed in order). Every wait is bounded; a timeout raises
+// `abort`, which every wave checks, so the workgroup always drains.
 //
 // The recurrence masks each cell's result to +0 at non-FLUID cells (zm) and
 // the factor sweep stores cx = cy = +0 there, so a neighbour the reference
 // skips contributes exactly cx*(+0) = +0, the same as a skipped term.
 constexpr int kBlk = 8;
-constexpr int kLoaders = 2;
-constexpr int kWaves = 6;
-enum { kWaveCompute = 0, kWaveWriter = 1, kWaveLoader0 = 2, kWaveIdle = 4, kWavePoller = 5 };
+constexpr int kMaxLoaders = 4;
+constexpr int kWaves = 8;
+enum { kWaveCompute = 0, kWaveWriter = 1, kWavePoller = 5, kWaveDot = 7 };
 constexpr int kERing = 512;  // edge ring, in steps
 constexpr int kMaxIn = 6;
 constexpr int kMaxOut = 6;
@@ -82,15 +87,26 @@ constexpr long kLdsSpin = 1L << 22;
 
 enum { SW_FWD = 0, SW_BWD = 1, SW_PRECON = 2 };
 
-// The first eight counters are what wave 0 polls; they are read together
-// (two 16-byte LDS reads, one wait).
+// waves 2, 3, 6 and, but for the backward sweep's dot wave, 7 are loaders
+constexpr int loaders(int kind) { return kind == SW_BWD ? 3 : 4; }
+template <int KIND>
+IFL_DEV int loader_of_wave(int w) {
+    const int k = (w & 2) ? (w >> 2) * 2 + (w & 1) : -1;
+    return k < loaders(KIND) ? k : -1;
+}
+
+// Wave 0 polls one pair per block: the counter of the loader that streams the
+// block and the edge counter, in one 8-byte LDS read.
 struct __align__(16) RingHdr {
-    int ready[kLoaders];   // per loader: 1 + last block published
-    int edge_ready;        // steps whose incoming edge value is in the edge ring
+    struct {
+        int ready;  // loader k: 1 + last block published
+        int edge;   // blocks whose incoming edge values are in the edge ring (the same in every pair)
+    } in[kMaxLoaders];
     int abort;
     int consumed;          // blocks whose slot is free again (writer)
     int computed;          // blocks wave 0 has finished (wave 0)
-    int pad[12 - kLoaders];
+    int dotted;            // backward sweep: blocks the dot wave has read
+    int pad[12 - 2 * kMaxLoaders];
 };
 static_assert(sizeof(RingHdr) == 64, "RingHdr layout");
 
@@ -99,7 +115,7 @@ struct StreamArgs {
     const void* in[kMaxIn];
     const uint64_t* fmask;
     double* edge;           // this sweep's edge buffers (nstrips * W)
-    void* out[kMaxOut];     // fwd: y, r   bwd: z   precon: precon, cx, cy (+ their single-precision copies)
+    void* out[kMaxOut];     // fwd: y, r (the loaders)   bwd: z   precon: precon, cx, cy (+ their single-precision copies)
     double* partial;
     PcgState* st;
     int* timeout;
@@ -120,45 +136,34 @@ struct StreamArgs {
 // and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima).
 #define IFL_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (0x7 << 4) | (0xF << 8) | (((n) >> 4) << 14))
 
-typedef __attribute__((address_space(3))) char lds_char;
-
 // LDS counters are read and written through inline asm: the compiler would
 // otherwise wait for every in-flight LDS-DMA load (vmcnt(0)) before any LDS
 // instruction in the loaders, and it must not move ring accesses across a
 // counter access in any wave ("memory" clobber).
-IFL_DEV unsigned lds_off(const void* p) { return (unsigned)(size_t)(const __attribute__((address_space(3))) char*)p; }
-IFL_DEV int lds_ld(const int* p) {
+// The header sits at the start of the workgroup's dynamic LDS; its fields are
+// addressed by their LDS byte offsets (a generic pointer would cost a null
+// check at every use).
+extern __shared__ __align__(16) char sweep_smem[];
+IFL_DEV unsigned smem_off() { return (unsigned)(size_t)(const __attribute__((address_space(3))) char*)sweep_smem; }
+#define IFL_HDR(field) (smem_off() + (unsigned)offsetof(RingHdr, field))
+IFL_DEV unsigned hdr_ready(int k) { return IFL_HDR(in) + 8u * (unsigned)k; }
+IFL_DEV unsigned hdr_edge(int k) { return IFL_HDR(in) + 8u * (unsigned)k + 4u; }
+IFL_DEV int lds_ld(unsigned off) {
     int v;
-    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(lds_off(p)) : "memory");
+    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(off) : "memory");
     return __builtin_amdgcn_readfirstlane(v);
 }
-// ready[0..4], edge_ready, abort, consumed of `h`, wave-uniform
-IFL_DEV void lds_ld8(const RingHdr* h, int (&c)[8]) {
-    typedef int v4i __attribute__((ext_vector_type(4)));
-    v4i lo, hi;
-    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:16\n\ts_waitcnt lgkmcnt(0)"
-                 : "=v"(lo), "=v"(hi)
-                 : "v"(lds_off(h))
-                 : "memory");
-    c[0] = __builtin_amdgcn_readfirstlane(lo.x);
-    c[1] = __builtin_amdgcn_readfirstlane(lo.y);
-    c[2] = __builtin_amdgcn_readfirstlane(lo.z);
-    c[3] = __builtin_amdgcn_readfirstlane(lo.w);
-    c[4] = __builtin_amdgcn_readfirstlane(hi.x);
-    c[5] = __builtin_amdgcn_readfirstlane(hi.y);
-    c[6] = __builtin_amdgcn_readfirstlane(hi.z);
-    c[7] = __builtin_amdgcn_readfirstlane(hi.w);
+IFL_DEV void lds_st(unsigned off, int v) {
+    asm volatile("ds_write_b32 %0, %1" : : "v"(off), "v"(v) : "memory");
 }
-IFL_DEV void lds_st(int* p, int v) {
-    asm volatile("ds_write_b32 %0, %1" : : "v"(lds_off(p)), "v"(v) : "memory");
-}
-// Spin until *p > bound; false on abort or timeout (which raises abort).
-IFL_DEV bool lds_wait_gt(const int* p, int bound, RingHdr* hdr, int* gtimeout) {
+// Spin until the counter at `off` exceeds `bound`; false on abort or timeout
+// (which raises abort).
+IFL_DEV bool lds_wait_gt(unsigned off, int bound, int* gtimeout) {
     long spins = 0;
-    while (lds_ld(p) <= bound) {
-        if (lds_ld(&hdr->abort)) return false;
+    while (lds_ld(off) <= bound) {
+        if (lds_ld(IFL_HDR(abort))) return false;
         if (++spins > kLdsSpin) {
-            lds_st(&hdr->abort, 1);
+            lds_st(IFL_HDR(abort), 1);
             atomicOr(gtimeout, 1);
             return false;
         }
@@ -239,8 +244,7 @@ IFL_DEV const const_u64* strip_masks(const StreamArgs& a, int j) {
 }
 
 // Each loader streams blocks k, k + kLoaders, ... with non-temporal loads
-// (every byte is read once per sweep; measured at 2048^2 with the writer's
-// non-temporal block stores: -40 us per backward sweep). Up to R blocks are in
+// (every byte is read once per sweep). Up to R blocks are in
 // flight in its registers (global_load_dwordx4: lane i holds bytes
 // [16 i, 16 i + 16) of each 1 KB run of an array's block), so the prefetch
 // depth does not depend on free LDS slots; a block is written into its slot
@@ -248,9 +252,10 @@ IFL_DEV const const_u64* strip_masks(const StreamArgs& a, int j) {
 // (MODE 1) the loader forms r + q*(-alpha) (scaledAdd 7:870; at FLUID cells
 // only from level 6 on) and keeps only the result.
 template <int KIND, int MODE, int LV, int NG, typename T>
-IFL_DEV void loader_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int k, int lane, long sbase, int nblk, int j) {
+IFL_DEV void loader_wave(const StreamArgs& a, char* ring, int k, int lane, long sbase, int nblk, int j) {
     typedef SweepShape<KIND, MODE, NG, T> S;
     constexpr int R = S::R, NL = S::NLD;
+    constexpr int kLoaders = loaders(KIND);
     constexpr bool UPD = KIND == SW_FWD && MODE >= 1;
     const int cols = a.sk.cols;
     const int nmine = nblk > k ? (nblk - k + kLoaders - 1) / kLoaders : 0;
@@ -260,7 +265,12 @@ IFL_DEV void loader_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int k, i
     vec4i b0[NL], b1[NL], b2[NL];
     // the FLUID masks the residual update needs (levels 6+), loaded with the
     // block so that their latency is hidden like the block's
-    constexpr bool MASKED = UPD && LV >= 6;
+    constexpr bool MASKED = KIND == SW_FWD && LV >= 6;
+    const int W = a.sk.W, H = a.sk.H;
+    // the mixed form's pressure solves keep r less its mean over FLUID cells;
+    // the convergence test reads r itself
+    const double r0 = KIND == SW_FWD && sizeof(T) == 4 ? a.st->rmean : 0.0;
+    double rmax = 0.0;
     uint64_t w0[4], w1[4], w2[4];
     auto issue = [&](int i, vec4i* B, uint64_t* WM) __attribute__((always_inline)) {
         const int col0 = block_col0<KIND>(k + i * kLoaders, cols);
@@ -286,42 +296,47 @@ IFL_DEV void loader_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int k, i
     auto stage = [&](int i, vec4i* B, uint64_t* WM) __attribute__((always_inline)) -> bool {
         if (i >= nmine) return true;
         const int b = k + i * kLoaders;
-        if (UPD && S::es(0) == 8) {
+        if (KIND == SW_FWD) {
+            // the residual: scaledAdd(_r, z, -alpha) 7:870, infinityNorm(_r)
+            // 7:871 (masked in 6+), and the new residual's store, all on the
+            // registers that hold the block
+            const int col0 = block_col0<KIND>(b, cols);
+            const long e0 = sbase + (long)col0 * kStrip;
+            constexpr int EL = 16 / S::es(0);  // elements per lane of a 1 KB run
+            typedef typename std::conditional<S::es(0) == 8, double, float>::type E;
+            const E an = S::es(0) == 8 ? (E)alpha_neg : (E)alpha_neg_f;
 #pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const vec2d r = __builtin_bit_cast(vec2d, B[m]);
-                vec2d rn = r + __builtin_bit_cast(vec2d, B[S::lo(4) + m]) * alpha_neg;
-                if (MASKED) {
-                    const unsigned bits = (unsigned)(WM[m] >> (2 * (lane & 31)));
-                    rn.x = (bits & 1u) ? rn.x : r.x;
-                    rn.y = (bits & 2u) ? rn.y : r.y;
+            for (int m = 0; m < S::rb(0) / 1024; m++) {
+                typedef E vecE __attribute__((ext_vector_type(EL)));
+                const vecE r = __builtin_bit_cast(vecE, B[m]);
+                vecE rn = r;
+                if (UPD) rn = r + __builtin_bit_cast(vecE, B[S::lo(UPD ? 4 : 0) + m]) * an;
+                // element EL*lane + c of run m: row and column inside the block
+                const int row0 = (EL * lane) & 63, col = EL * m + ((EL * lane) >> 6);
+                const unsigned bits = MASKED ? (unsigned)(WM[m] >> row0) : 0;
+#pragma unroll
+                for (int c = 0; c < EL; c++) {
+                    const int row = row0 + c;
+                    const bool take = MASKED ? ((bits >> c) & 1u) != 0
+                                             : j * kStrip + row < H && (unsigned)(col0 + col - row) < (unsigned)W;
+                    if (MASKED) rn[c] = take ? rn[c] : r[c];
+                    const double rv = (double)rn[c];
+                    const double mx = smax(rmax, fabs(sizeof(T) == 4 ? rv + r0 : rv));
+                    rmax = take ? mx : rmax;
                 }
                 B[m] = __builtin_bit_cast(vec4i, rn);
-            }
-        } else if (UPD) {
-            typedef float vec4f __attribute__((ext_vector_type(4)));
-#pragma unroll
-            for (int m = 0; m < 2; m++) {
-                const vec4f r = __builtin_bit_cast(vec4f, B[m]);
-                vec4f rn = r + __builtin_bit_cast(vec4f, B[S::lo(4) + m]) * alpha_neg_f;
-                if (MASKED) {
-                    const unsigned bits = (unsigned)(WM[m] >> (4 * (lane & 15)));
-                    rn.x = (bits & 1u) ? rn.x : r.x;
-                    rn.y = (bits & 2u) ? rn.y : r.y;
-                    rn.z = (bits & 4u) ? rn.z : r.z;
-                    rn.w = (bits & 8u) ? rn.w : r.w;
-                }
-                B[m] = __builtin_bit_cast(vec4i, rn);
+                if (UPD) __builtin_nontemporal_store(B[m], (vec4i*)((char*)a.out[1] + e0 * S::es(0) + m * 1024 + lane * 16));
             }
         }
-        if (!lds_wait_gt(&hdr->consumed, b - a.nb, hdr, a.timeout)) return false;
+        if (!lds_wait_gt(IFL_HDR(consumed), b - a.nb, a.timeout)) return false;
+        if (KIND == SW_BWD && !lds_wait_gt(IFL_HDR(dotted), b - a.nb, a.timeout)) return false;
         char* slot = ring + (long)(b % a.nb) * a.slot_bytes;
 #pragma unroll
         for (int ai = 0; ai < S::NS; ai++)
 #pragma unroll
             for (int m = 0; m < S::rb(ai) / 1024; m++)
                 *(vec4i*)(slot + S::ro(ai) + m * 1024 + lane * 16) = B[S::lo(ai) + m];
-        lds_st(&hdr->ready[k], b + 1);
+        lds_st(hdr_ready(k), b + 1);
         if (i + R < nmine) issue(i + R, B, WM);
         return true;
     };
@@ -333,16 +348,20 @@ IFL_DEV void loader_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int k, i
         if (R > 1 && !stage(i + 1, b1, w1)) return;
         if (R > 2 && !stage(i + 2, b2, w2)) return;
     }
+    if (KIND == SW_FWD) {
+        rmax = wave_max(rmax);
+        if (lane == 0) atomicMax((unsigned long long*)&a.st->max_err, (unsigned long long)as_bits(rmax));
+    }
 }
 
 // Strips without a neighbour on the input side get +0 edges.
 template <int KIND>
-IFL_DEV void poller_wave(const StreamArgs& a, const double* ein, double* ering, RingHdr* hdr, int lane) {
+IFL_DEV void poller_wave(const StreamArgs& a, const double* ein, double* ering, int lane) {
     const int cols = a.sk.cols, W = a.sk.W;
     int t0 = 0;
     long spins = 0;
     // ring capacity: the edges of finished blocks are no longer read
-    int cap = lds_ld(&hdr->computed) * kBlk + kERing;
+    int cap = lds_ld(IFL_HDR(computed)) * kBlk + kERing;
     while (t0 < cols) {
         const int t = t0 + lane;
         const int x = edge_x<KIND>(t, cols);
@@ -351,8 +370,8 @@ IFL_DEV void poller_wave(const StreamArgs& a, const double* ein, double* ering, 
         uint64_t v = need ? ld_relaxed(ein + x) : 0;
         // while the load is in flight: the abort flag, and the capacity for
         // the next round (read before that round's load: never too large)
-        const int ab = lds_ld(&hdr->abort);
-        const int cap_next = lds_ld(&hdr->computed) * kBlk + kERing;
+        const int ab = lds_ld(IFL_HDR(abort));
+        const int cap_next = lds_ld(IFL_HDR(computed)) * kBlk + kERing;
         if (ab) return;
         const bool ok = inwin && (!need || v != kSentinel);
         const uint64_t m = __ballot(ok);
@@ -361,14 +380,15 @@ IFL_DEV void poller_wave(const StreamArgs& a, const double* ein, double* ering, 
         cap = cap_next;
         if (n > 0) {
             t0 += n;
-            lds_st(&hdr->edge_ready, t0);
+#pragma unroll
+            for (int k = 0; k < loaders(KIND); k++) lds_st(hdr_edge(k), t0 / kBlk);
             spins = 0;
         } else {
             // no sleep: each poll is a memory round trip already, and the
             // sooner a value is seen the sooner this strip moves (measured at
             // 2048^2: -12 us per forward sweep, -20 us per backward sweep)
             if (++spins > kLdsSpin) {
-                lds_st(&hdr->abort, 1);
+                lds_st(IFL_HDR(abort), 1);
                 atomicOr(a.timeout, 1);
                 return;
             }
@@ -383,15 +403,16 @@ IFL_DEV void poller_wave(const StreamArgs& a, const double* ein, double* ering, 
     }
 }
 
-// Wave 0. Operand registers are double-buffered by block (8 steps): a block
-// first issues the LDS reads of the next block, then runs its steps (against
-// half-block buffers: 382 / 371 us instead of 408 / 416 us per forward /
-// backward sweep at 2048^2, with the trace stamps compiled out).
+// Wave 0. Operand registers are double-buffered by block (8 steps): while a
+// block's steps run, the LDS reads of the next block go out between them.
+// One strip alone with nothing to wait for, 2112 steps: 94 us with the reads
+// at the block's start, the whole step formed in one chain and several exits
+// from the readiness check; 76 us as it is now.
 // TR: the diagnostic build with per-block time stamps (ifl_debug_trace_sweep);
 // the stamps' branches cost ~6 % of a sweep, so the solver's own sweeps are
 // built without them.
 template <int KIND, int MODE, int NG, typename T, bool TR>
-IFL_DEV void compute_wave(const StreamArgs& a, char* ring, RingHdr* hdr, const double* ering, int j, int lane) {
+IFL_DEV void compute_wave(const StreamArgs& a, char* ring, const double* ering, int j, int lane) {
     typedef SweepShape<KIND, MODE, NG, T> S;
     typedef typename Vec2<T>::type V2;
     constexpr int NT = S::NT;
@@ -403,33 +424,37 @@ IFL_DEV void compute_wave(const StreamArgs& a, char* ring, RingHdr* hdr, const d
         if (TR && lane == 0) tr[b * kTraceStamps + i] = __builtin_amdgcn_s_memrealtime();
     };
 
-    // Readiness is cached: the counters are re-read only when the cached
-    // limit does not cover the request. Loader k has published blocks
-    // k, k + kLoaders, ..., ready[k] - 1, so every block below the smallest
-    // "next block" over the loaders is in the ring.
-    int block_limit = 0, edge_limit = 0;
-    // true once block b is in the ring and the edges of steps < tend are in
-    // the edge ring
-    auto ready = [&](int b, int tend) -> bool {
-        if (b < block_limit && tend <= edge_limit) return true;
-        long spins = 0;
-        while (true) {
-            int c[8];
-            lds_ld8(hdr, c);
-            int lim = 1 << 30;
-#pragma unroll
-            for (int k = 0; k < kLoaders; k++) lim = min(lim, c[k] == 0 ? k : c[k] - 1 + kLoaders);
-            block_limit = lim;
-            edge_limit = c[kLoaders];
-            if (b < block_limit && tend <= edge_limit) return true;
-            if (c[kLoaders + 1]) return false;  // abort
-            if (++spins > kLdsSpin) {
-                lds_st(&hdr->abort, 1);
+    // Block b can be loaded once its loader has published it and the edges of
+    // its steps are in the edge ring (earlier blocks were checked before it).
+    // The pair of counters is read ahead, during the block before, so that in
+    // the usual case the check costs no LDS round trip. Past the last block
+    // the last block's counters are read again. The check has one exit: with
+    // returns inside the loop the branches around every block cost more than
+    // a step.
+    typedef uint64_t __attribute__((address_space(3))) lds_u64;
+    auto peek = [&](int b) -> uint64_t {
+        const int bm = b < nblk ? b : nblk - 1;
+        return __hip_atomic_load((lds_u64*)(uintptr_t)hdr_ready(bm % loaders(KIND)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    auto limit = [&](uint64_t c) { return __builtin_amdgcn_readfirstlane(min((int)c, (int)(c >> 32))); };
+    bool stop = false;
+    auto ready = [&](int b, uint64_t seen) {
+        const int bm = b < nblk ? b : nblk - 1;
+        if (__builtin_expect(limit(seen) <= bm, 0)) {
+            long spins = 0;
+            int ab = 0;
+            do {
+                seen = peek(b);
+                ab = lds_ld(IFL_HDR(abort));
+                spins++;
+            } while (limit(seen) <= bm && !ab && spins <= kLdsSpin);
+            stop = limit(seen) <= bm;
+            if (stop && !ab) {
+                lds_st(IFL_HDR(abort), 1);
                 atomicOr(a.timeout, 1);
-                return false;
             }
-            __builtin_amdgcn_s_sleep(1);
         }
+        asm volatile("" : : : "memory");
     };
 
     // Operands of a block, shaped as the loads deliver them so that the
@@ -449,27 +474,27 @@ IFL_DEV void compute_wave(const StreamArgs& a, char* ring, RingHdr* hdr, const d
     QV QA[NP], QB[NP];
     vec2d EA[NP], EB[NP];
     vec4u MA0, MA1, MB0, MB1;
-    auto load_blk = [&](const char* slot, int b, V2 (&X)[NT][NP], QV (&Q)[NP], vec2d (&E)[NP], vec4u& M0, vec4u& M1) {
-        const int bm = b < nblk ? b : nblk - 1;
-        // a block's 8 edges are contiguous in the ring (8 divides its size)
-        const double* eb = ering + ((unsigned)(bm * kBlk) & (unsigned)(kERing - 1));
-#pragma unroll
-        for (int p = 0; p < NP; p++) {
-            const int e0 = step_in_block<KIND>(2 * p) * kStrip + lane;
-            const int e1 = step_in_block<KIND>(2 * p + 1) * kStrip + lane;
-#pragma unroll
-            for (int i = 0; i < NT; i++) {
-                const T* arr = (const T*)(slot + S::ro(S::tarr(i)));
-                X[i][p].x = arr[e0];
-                X[i][p].y = arr[e1];
-            }
-            if (KIND == SW_FWD) {
-                const QE* arr = (const QE*)slot;
-                Q[p].x = arr[e0];
-                Q[p].y = arr[e1];
-            }
+    // item q of a block's loads: pair q / PERP, then its arrays and its edges
+    constexpr int PERP = NT + (KIND == SW_FWD ? 2 : 1), NI = NP * PERP;
+    auto load_item = [&](int q, const char* slot, int bm, V2 (&X)[NT][NP], QV (&Q)[NP], vec2d (&E)[NP]) __attribute__((always_inline)) {
+        const int p = q / PERP, i = q % PERP;
+        const int e0 = step_in_block<KIND>(2 * p) * kStrip + lane;
+        const int e1 = step_in_block<KIND>(2 * p + 1) * kStrip + lane;
+        if (i < NT) {
+            const T* arr = (const T*)(slot + S::ro(S::tarr(i)));
+            X[i][p].x = arr[e0];
+            X[i][p].y = arr[e1];
+        } else if (KIND == SW_FWD && i == NT) {
+            const QE* arr = (const QE*)slot;
+            Q[p].x = arr[e0];
+            Q[p].y = arr[e1];
+        } else {
+            // a block's 8 edges are contiguous in the ring (8 divides its size)
+            const double* eb = ering + ((unsigned)(bm * kBlk) & (unsigned)(kERing - 1));
             E[p] = *(const vec2d*)(eb + 2 * p);
         }
+    };
+    auto load_masks = [&](int bm, vec4u& M0, vec4u& M1) __attribute__((always_inline)) {
         const int c0 = block_col0<KIND>(bm, cols);  // the block's 8 columns, lowest first
         M0 = *(const const_u64x4*)(fm + c0);
         M1 = *(const const_u64x4*)(fm + c0 + 4);
@@ -481,53 +506,82 @@ IFL_DEV void compute_wave(const StreamArgs& a, char* ring, RingHdr* hdr, const d
         return c == 0 ? M.x : c == 1 ? M.y : c == 2 ? M.z : M.w;
     };
     T Pw = 0, Pn = 0, zs = 0;
+    uint64_t seen = 0;  // the counters of the block after next
     auto run_blk = [&](const char* slot, int b, const V2 (&X)[NT][NP], const QV (&Q)[NP], const vec2d (&E)[NP],
                        const vec4u& M0, const vec4u& M1, const char* nslot, V2 (&Y)[NT][NP], QV (&P)[NP],
                        vec2d (&F)[NP], vec4u& N0, vec4u& N1) {
         T* out = (T*)(slot + S::OUT);
+        const int bm = b + 1 < nblk ? b + 1 : nblk - 1;
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-        load_blk(nslot, b + 1, Y, P, F, N0, N1);
+        load_masks(bm, N0, N1);
         __builtin_amdgcn_sched_barrier(0);
+        // The next block's loads go out three per step, in the order of use, so
+        // that each step's chain hides them and the last step hides the last
+        // loads' latency.
+        constexpr int PER = (NI + kBlk - 2) / (kBlk - 1);
+        auto x = [&](int i, int k) -> T { return (k & 1) ? X[i][k >> 1].y : X[i][k >> 1].x; };
+        auto rq = [&](int k) -> T { return (T)((k & 1) ? Q[k >> 1].y : Q[k >> 1].x); };
+        // the part of a step that needs only this row's last result, formed
+        // one step ahead: the chain between rows then starts with the lane
+        // move (a one-wave loop of the steps alone: 52 -> 37 clocks per step)
+        T t1 = 0;
+        if (KIND == SW_FWD) t1 = rq(0) - Pw;
+        if (KIND == SW_BWD) t1 = x(0, 0) - x(1, 0) * zs;
+        T zlast = 0;
 #pragma unroll
         for (int k = 0; k < kBlk; k++) {
             const int e = step_in_block<KIND>(k) * kStrip + lane;
             const bool f = lane_on(mask_of(M0, M1, k));
-            const int p = k >> 1;
-            const bool hi = k & 1;
-            auto x = [&](int i) -> T { return hi ? X[i][p].y : X[i][p].x; };
-            const T ek = (T)(hi ? E[p].y : E[p].x);
+            const T ek = (T)((k & 1) ? E[k >> 1].y : E[k >> 1].x);
+            T zk;
             if (KIND == SW_FWD) {
                 const T Ps = lane_shr1(Pn, ek);
-                const T t1 = (T)(hi ? Q[p].y : Q[p].x) - Pw;
+                __builtin_amdgcn_sched_barrier(0);
                 const T tt = t1 - Ps;
-                const T zz = tt * x(2);
-                const T zm = f ? zz : (T)0;
-                Pw = x(0) * zm;
-                Pn = x(1) * zm;
-                out[e] = zm;
+                const T zz = tt * x(2, k);
+                zk = f ? zz : (T)0;
+                __builtin_amdgcn_sched_barrier(0);
+                Pn = x(1, k) * zk;
+                __builtin_amdgcn_sched_barrier(0);
+                if (k + 1 < kBlk)
+                    t1 = rq(k + 1) - x(0, k) * zk;
+                else
+                    Pw = x(0, k) * zk;
             } else if (KIND == SW_BWD) {
                 const T zn = lane_shl1(zs, ek);
-                const T t1 = x(0) - x(1) * zs;
-                const T tt = t1 - x(2) * zn;
-                const T zz = tt * x(3);
-                zs = f ? zz : (T)0;
-                out[e] = zs;
+                __builtin_amdgcn_sched_barrier(0);
+                const T tt = t1 - x(2, k) * zn;
+                const T zz = tt * x(3, k);
+                zs = zk = f ? zz : (T)0;
+                __builtin_amdgcn_sched_barrier(0);
+                if (k + 1 < kBlk) t1 = x(0, k + 1) - x(1, k + 1) * zs;
             } else {
                 const double Ns = lane_shr1((double)Pn, (double)ek);
-                const double ad = x(0);
+                const double ad = x(0, k);
                 double ev = ad;
                 ev = ev - Pw;
                 ev = ev - Ns;
                 if (ev < sigma * ad) ev = ad;
                 const double pcv = 1.0 / sqrt(ev);
-                const double px = x(1) * pcv;
-                const double py = x(2) * pcv;
+                const double px = x(1, k) * pcv;
+                const double py = x(2, k) * pcv;
                 const double eo = px * px + tau * px * py;
                 const double no = py * py + tau * px * py;
                 Pw = f ? eo : 0.0;
                 Pn = f ? no : 0.0;
-                out[e] = pcv;
+                zk = pcv;
             }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = k * PER; q < (k + 1) * PER && q < NI; q++) load_item(q, nslot, bm, Y, P, F);
+            if (k == kBlk - 2) seen = peek(b + 2);
+            // two steps' results in one LDS instruction
+            if (k & 1) {
+                out[step_in_block<KIND>(k - 1) * kStrip + lane] = zlast;
+                out[e] = zk;
+            }
+            zlast = zk;
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     {
@@ -535,53 +589,53 @@ IFL_DEV void compute_wave(const StreamArgs& a, char* ring, RingHdr* hdr, const d
         const vec4u m = *(const const_u64x4*)(fm + c0);
         asm volatile("" : : "s"(m.x));
     }
-    if (!ready(0, kBlk)) return;
-    const char* slot = ring;  // block 0 is in slot 0
-    load_blk(slot, 0, XA, QA, EA, MA0, MA1);
-    int sidx = 0;
-    auto next_slot = [&]() {
-        sidx = sidx + 1 == a.nb ? 0 : sidx + 1;
-        return ring + (long)sidx * a.slot_bytes;
-    };
+    ready(0, peek(0));
+    if (stop) return;
+    load_masks(0, MA0, MA1);
+#pragma unroll
+    for (int q = 0; q < NI; q++) load_item(q, ring, 0, XA, QA, EA);
+    seen = peek(1);
+    const int ring_bytes = a.nb * a.slot_bytes;
+    int off = 0;  // block 0 is in slot 0
+    // nblk is even (cols is a multiple of 16)
     for (int b = 0; b < nblk; b += 2) {
         // block b from A; block b+1 goes to B
         stamp(b, 0);
-        if (b + 1 < nblk && !ready(b + 1, (b + 2) * kBlk)) return;
+        ready(b + 1, seen);
+        if (stop) break;
         stamp(b, 1);
-        const char* nslot = next_slot();
-        run_blk(slot, b, XA, QA, EA, MA0, MA1, nslot, XB, QB, EB, MB0, MB1);
-        lds_st(&hdr->computed, b + 1);
+        int noff = off + a.slot_bytes;
+        noff = noff == ring_bytes ? 0 : noff;
+        run_blk(ring + off, b, XA, QA, EA, MA0, MA1, ring + noff, XB, QB, EB, MB0, MB1);
+        lds_st(IFL_HDR(computed), b + 1);
         stamp(b, 4);
-        slot = nslot;
-        if (b + 1 >= nblk) break;
+        off = noff;
         stamp(b + 1, 0);
-        if (b + 2 < nblk && !ready(b + 2, (b + 3) * kBlk)) return;
+        ready(b + 2, seen);
+        if (stop) break;
         stamp(b + 1, 1);
-        nslot = next_slot();
-        run_blk(slot, b + 1, XB, QB, EB, MB0, MB1, nslot, XA, QA, EA, MA0, MA1);
-        lds_st(&hdr->computed, b + 2);
+        noff = off + a.slot_bytes;
+        noff = noff == ring_bytes ? 0 : noff;
+        run_blk(ring + off, b + 1, XB, QB, EB, MB0, MB1, ring + noff, XA, QA, EA, MA0, MA1);
+        lds_st(IFL_HDR(computed), b + 2);
         stamp(b + 1, 4);
-        slot = nslot;
+        off = noff;
     }
 }
 
 // The writer wave: drains finished blocks.
 template <int KIND, int MODE, int LV, int NG, typename T, bool TR>
-IFL_DEV void writer_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int j, int lane, double* eout) {
+IFL_DEV void writer_wave(const StreamArgs& a, char* ring, int j, int lane, double* eout) {
     typedef SweepShape<KIND, MODE, NG, T> S;
-    constexpr bool VM = LV >= 6;   // vector operations masked to FLUID cells
-    constexpr bool AUX = LV == 4;  // levels 4-5: the dot reads the reference's _z at non-FLUID cells
-    const int W = a.sk.W, H = a.sk.H, cols = a.sk.cols, nblk = cols / kBlk;
+    // outputs stored step by step: the factor, the stage form's masked _z and
+    // the mixed form's widened _z
+    constexpr bool PER_STEP = KIND == SW_PRECON || (KIND == SW_BWD && (MODE == 0 || (MODE == 1 && sizeof(T) != 8)));
+    const int W = a.sk.W, cols = a.sk.cols, nblk = cols / kBlk;
     const const_u64* fm = strip_masks(a, j);
     const long sbase = (long)j * a.sk.strip_sz;
-    const bool row_ok = j * kStrip + lane < H;
     const double tau = a.tau;
-    // the mixed form's pressure solves keep r less its mean over FLUID cells;
-    // the convergence test reads r itself
-    const double r0 = KIND == SW_FWD && sizeof(T) == 4 ? a.st->rmean : 0.0;
-    double rmax = 0.0, acc = 0.0, zsum = 0.0;
     for (int b = 0; b < nblk; b++) {
-        if (!lds_wait_gt(&hdr->computed, b, hdr, a.timeout)) return;
+        if (!lds_wait_gt(IFL_HDR(computed), b, a.timeout)) return;
         char* slot = ring + (long)(b % a.nb) * a.slot_bytes;
         auto in = [&](int ai) { return slot + S::ro(ai); };  // region of streamed array ai
         const T* out = (const T*)(slot + S::OUT);
@@ -626,7 +680,7 @@ IFL_DEV void writer_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int j, i
                 st_relaxed(eout + x, as_bits(v));
             }
         }
-        if (KIND != SW_PRECON) {
+        if (KIND == SW_BWD && MODE == 0) {
 #pragma unroll
             for (int k = 0; k < kBlk; k++) M[k] = fm[col0 + k];
         }
@@ -635,23 +689,13 @@ IFL_DEV void writer_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int j, i
         // recurrence, on another SIMD of the CU, measurably slows down while
         // this wave runs branchy code or masked stores).
 #pragma unroll
-        for (int k = 0; k < kBlk; k++) {
+        for (int k = 0; k < (PER_STEP ? kBlk : 0); k++) {
             const int t = b * kBlk + k;
             const int c = step_col<KIND>(t, cols);
             const int e = step_in_block<KIND>(k) * kStrip + lane;
-            const int x = c - lane;
-            const bool valid = row_ok && x >= 0 && x < W;
-            const bool f = lane_on(M[c - col0]);
-            const bool take = VM ? f : valid;
-            if (KIND == SW_FWD) {
-                // infinityNorm(_r) 7:871 (masked in 6+) of the residual the sweep used
-                const double rv = MODE == 2 ? (double)((const T*)in(0))[e] : ((const double*)in(0))[e];
-                const double m = smax(rmax, fabs(sizeof(T) == 4 ? rv + r0 : rv));
-                rmax = take ? m : rmax;
-            } else if (KIND == SW_BWD) {
-                // _z (wave 0 left +0 at non-FLUID cells); dotProduct(_z, _r)
-                // 7:880 (unmasked in 3-5, where the reference's _z is A s at
-                // non-FLUID cells)
+            const bool f = KIND == SW_PRECON || MODE == 0 ? lane_on(M[c - col0]) : true;
+            if (KIND == SW_BWD) {
+                // _z (wave 0 left +0 at non-FLUID cells)
                 const double zz = (double)out[e];
                 if (MODE == 0) {
                     // the stage form keeps _z at non-FLUID cells as it was
@@ -665,13 +709,6 @@ IFL_DEV void writer_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int j, i
                     // from the second read of the block from LDS)
                     ((double*)a.out[0])[gblk + e] = zz;
                 }
-                const double rv = MODE == 2 ? (double)((const T*)in(4))[e] : ((const double*)in(4))[e];
-                const double aux = !AUX ? 0.0 : MODE == 2 ? (double)((const T*)in(5))[e] : ((const double*)in(5))[e];
-                const double zdot = f ? zz : aux;
-                const double na = acc + zdot * rv;
-                acc = take ? na : acc;
-                if (MODE == 2 || sizeof(T) == 4)
-                    zsum = f ? zsum + zz : zsum;  // the mean taken off z (deflation)
             } else {
                 // the factor at FLUID cells; cx = aPlusX*precon, cy likewise, +0 elsewhere
                 const double pcv = (double)out[e];
@@ -697,7 +734,6 @@ IFL_DEV void writer_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int j, i
         };
         if (KIND == SW_FWD) {
             store_block(a.out[0], (const char*)out, sizeof(T));
-            if (MODE >= 1) store_block(a.out[1], in(0), S::es(0));
         } else if (KIND == SW_BWD) {
             if ((MODE == 1 && sizeof(T) == 8) || MODE == 2) store_block(a.out[0], (const char*)out, sizeof(T));
         } else if (KIND == SW_PRECON) {
@@ -705,34 +741,73 @@ IFL_DEV void writer_wave(const StreamArgs& a, char* ring, RingHdr* hdr, int j, i
             store_block(a.out[2], in(2), 8);
         }
         if (TR && lane == 0) a.trace[((long)j * nblk + b) * kTraceStamps + 5] = __builtin_amdgcn_s_memrealtime();
-        lds_st(&hdr->consumed, b + 1);
+        lds_st(IFL_HDR(consumed), b + 1);
     }
-    if (KIND == SW_FWD) {
-        rmax = wave_max(rmax);
-        if (lane == 0) atomicMax((unsigned long long*)&a.st->max_err, (unsigned long long)as_bits(rmax));
-    } else if (KIND == SW_BWD) {
-        acc = wave_sum(acc);
-        if (lane == 0) a.partial[j] = acc;
-        if (MODE == 2 || sizeof(T) == 4) {
-            zsum = wave_sum(zsum);
-            if (lane == 0) a.partial[a.sk.nstrips + j] = zsum;
+}
+
+// The backward sweep's dot wave: dotProduct(_z, _r) 7:880 of each finished
+// block in sweep order (unmasked in levels 3-5, where the reference's _z is
+// A s at non-FLUID cells), and the mixed form's sum of z. Straight-line: loads
+// first and selects instead of branches. On the writer, whose ~250
+// instructions per block it doubled, it set the pace of the whole sweep
+// (2048^2: 0.45 us per block with nothing else to wait for).
+template <int MODE, int LV, int NG, typename T>
+IFL_DEV void dot_wave(const StreamArgs& a, const char* ring, int j, int lane) {
+    typedef SweepShape<SW_BWD, MODE, NG, T> S;
+    constexpr bool VM = LV >= 6;   // vector operations masked to FLUID cells
+    constexpr bool AUX = LV == 4;  // levels 4-5: the dot reads the reference's _z at non-FLUID cells
+    const int W = a.sk.W, cols = a.sk.cols, nblk = cols / kBlk;
+    const const_u64* fm = strip_masks(a, j);
+    const bool row_ok = j * kStrip + lane < a.sk.H;
+    double acc = 0.0, zsum = 0.0;
+    for (int b = 0; b < nblk; b++) {
+        const int col0 = block_col0<SW_BWD>(b, cols);
+        uint64_t M[kBlk];
+#pragma unroll
+        for (int k = 0; k < kBlk; k++) M[k] = fm[col0 + k];
+        if (!lds_wait_gt(IFL_HDR(computed), b, a.timeout)) return;
+        const char* slot = ring + (long)(b % a.nb) * a.slot_bytes;
+        const T* out = (const T*)(slot + S::OUT);
+        double zv[kBlk], rv[kBlk], av[kBlk];
+#pragma unroll
+        for (int k = 0; k < kBlk; k++) {
+            const int e = step_in_block<SW_BWD>(k) * kStrip + lane;
+            zv[k] = (double)out[e];
+            rv[k] = MODE == 2 ? (double)((const T*)(slot + S::ro(4)))[e] : ((const double*)(slot + S::ro(4)))[e];
+            av[k] = !AUX ? 0.0 : MODE == 2 ? (double)((const T*)(slot + S::ro(5)))[e] : ((const double*)(slot + S::ro(5)))[e];
         }
+#pragma unroll
+        for (int k = 0; k < kBlk; k++) {
+            const int x = step_col<SW_BWD>(b * kBlk + k, cols) - lane;
+            const bool f = lane_on(M[step_in_block<SW_BWD>(k)]);
+            const bool take = VM ? f : row_ok && x >= 0 && x < W;
+            const double na = acc + (VM || f ? zv[k] : av[k]) * rv[k];
+            acc = take ? na : acc;
+            if (MODE == 2 || sizeof(T) == 4)
+                zsum = f ? zsum + zv[k] : zsum;  // the mean taken off z (deflation)
+        }
+        lds_st(IFL_HDR(dotted), b + 1);
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) a.partial[j] = acc;
+    if (MODE == 2 || sizeof(T) == 4) {
+        zsum = wave_sum(zsum);
+        if (lane == 0) a.partial[a.sk.nstrips + j] = zsum;
     }
 }
 
 template <int KIND, int MODE, int LV, int NG, typename T, bool TR>
 IFL_DEV void sweep_body(const StreamArgs& a, int j) {
-    extern __shared__ __align__(16) char smem[];
+    char* smem = sweep_smem;
     PcgState* st = a.st;
     if (KIND != SW_PRECON && ((MODE >= 1 && st->done) || st->timeout)) return;
     // inside the PCG loop the backward sweep follows the convergence test
     // (7:872-876): it does nothing once max|r| < tol (a.sigma holds tol)
     if (KIND == SW_BWD && MODE == 1 && st->max_err < a.sigma) return;
-    RingHdr* hdr = (RingHdr*)smem;
     double* ering = (double*)(smem + sizeof(RingHdr));
     char* ring = smem + sizeof(RingHdr) + kERing * sizeof(double);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (threadIdx.x < (int)(sizeof(RingHdr) / sizeof(int))) ((int*)hdr)[threadIdx.x] = 0;
+    if (threadIdx.x < (int)(sizeof(RingHdr) / sizeof(int))) ((int*)smem)[threadIdx.x] = 0;
     __syncthreads();
 
     const int W = a.sk.W, nblk = a.sk.cols / kBlk;
@@ -744,13 +819,15 @@ IFL_DEV void sweep_body(const StreamArgs& a, int j) {
     double* eout = has_out ? a.edge + (long)(KIND == SW_BWD ? j : j + 1) * W : nullptr;
 
     if (wave == kWaveCompute)
-        compute_wave<KIND, MODE, NG, T, TR>(a, ring, hdr, ering, j, lane);
+        compute_wave<KIND, MODE, NG, T, TR>(a, ring, ering, j, lane);
     else if (wave == kWaveWriter)
-        writer_wave<KIND, MODE, LV, NG, T, TR>(a, ring, hdr, j, lane, eout);
+        writer_wave<KIND, MODE, LV, NG, T, TR>(a, ring, j, lane, eout);
     else if (wave == kWavePoller)
-        poller_wave<KIND>(a, ein, ering, hdr, lane);
-    else if (wave >= kWaveLoader0 && wave < kWaveLoader0 + kLoaders)
-        loader_wave<KIND, MODE, LV, NG, T>(a, ring, hdr, wave - kWaveLoader0, lane, sbase, nblk, j);
+        poller_wave<KIND>(a, ein, ering, lane);
+    else if (KIND == SW_BWD && wave == kWaveDot)
+        dot_wave<MODE, LV, NG, T>(a, ring, j, lane);
+    else if (loader_of_wave<KIND>(wave) >= 0)
+        loader_wave<KIND, MODE, LV, NG, T>(a, ring, loader_of_wave<KIND>(wave), lane, sbase, nblk, j);
 }
 
 // The sweep kernels that deal a launch's strips upstream first
