@@ -243,8 +243,12 @@ IFL_DEV const const_u64* strip_masks(const StreamArgs& a, int j) {
     return (const const_u64*)(uintptr_t)(a.fmask + (long)j * a.sk.cols);
 }
 
-// Each loader streams blocks k, k + kLoaders, ... with non-temporal loads
-// (every byte is read once per sweep). Up to R blocks are in
+// Each loader streams blocks k, k + kLoaders, ... with ordinary loads: one
+// CU streams 66 GB/s from HBM and 100 from the Infinity Cache with them, 59
+// and 56 with non-temporal ones, and what a sweep stores is read by the next
+// kernel (per PCG iteration: solver 7 at 2048^2 761 -> 747 us, at 1000x777
+// 317 -> 282, at 512^2 171 -> 163; the batch's launches 1-4 % faster). Up to
+// R blocks are in
 // flight in its registers (global_load_dwordx4: lane i holds bytes
 // [16 i, 16 i + 16) of each 1 KB run of an array's block), so the prefetch
 // depth does not depend on free LDS slots; a block is written into its slot
@@ -279,7 +283,7 @@ IFL_DEV void loader_wave(const StreamArgs& a, char* ring, int k, int lane, long 
         for (int ai = 0; ai < NG; ai++) {
             const char* p = (const char*)a.in[ai] + e0 * S::es(ai) + lane * 16;
 #pragma unroll
-            for (int m = 0; m < S::rb(ai) / 1024; m++) B[S::lo(ai) + m] = __builtin_nontemporal_load((const vec4i*)(p + m * 1024));
+            for (int m = 0; m < S::rb(ai) / 1024; m++) B[S::lo(ai) + m] = *(const vec4i*)(p + m * 1024);
         }
         if (MASKED && S::es(0) == 8) {
             // element 2*lane + c of run m is step 2m + lane/32, row 2*(lane%32) + c
@@ -325,7 +329,7 @@ IFL_DEV void loader_wave(const StreamArgs& a, char* ring, int k, int lane, long 
                     rmax = take ? mx : rmax;
                 }
                 B[m] = __builtin_bit_cast(vec4i, rn);
-                if (UPD) __builtin_nontemporal_store(B[m], (vec4i*)((char*)a.out[1] + e0 * S::es(0) + m * 1024 + lane * 16));
+                if (UPD) *(vec4i*)((char*)a.out[1] + e0 * S::es(0) + m * 1024 + lane * 16) = B[m];
             }
         }
         if (!lds_wait_gt(IFL_HDR(consumed), b - a.nb, a.timeout)) return false;
@@ -730,7 +734,7 @@ IFL_DEV void writer_wave(const StreamArgs& a, char* ring, int j, int lane, doubl
             char* d = (char*)dst + gblk * es + lane * 16;
 #pragma unroll
             for (int m = 0; m < 4; m++)
-                if (m * 1024 < 512 * es) __builtin_nontemporal_store(*(const vec4i*)(src + m * 1024 + lane * 16), (vec4i*)(d + m * 1024));
+                if (m * 1024 < 512 * es) *(vec4i*)(d + m * 1024) = *(const vec4i*)(src + m * 1024 + lane * 16);
         };
         if (KIND == SW_FWD) {
             store_block(a.out[0], (const char*)out, sizeof(T));
