@@ -267,6 +267,8 @@ void free_all(Solver* s) {
     if (s->step_flags_host) (void)hipHostFree(s->step_flags_host);
     flip_free(s);
     if (s->st_host) (void)hipHostFree(s->st_host);
+    for (hipEvent_t e : s->ev_group)
+        if (e) (void)hipEventDestroy(e);
     if (s->ev0) (void)hipEventDestroy(s->ev0);
     if (s->ev1) (void)hipEventDestroy(s->ev1);
     for (auto& t : s->timed) {
@@ -283,6 +285,7 @@ int init_solver(Solver* s) {
     IFL_HIP(hipSetDevice(s->device));
     IFL_TRY(scratch_init(s));
     IFL_HIP(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
+    for (hipEvent_t& e : s->ev_group) IFL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     IFL_HIP(hipEventCreate(&s->ev0));
     IFL_HIP(hipEventCreate(&s->ev1));
     int lds = 0;
@@ -357,8 +360,8 @@ int init_solver(Solver* s) {
     IFL_TRY(dalloc(s, &s->partial, s->npartial));
     IFL_HIP(hipMalloc((void**)&s->st, sizeof(PcgState)));
     IFL_HIP(hipMemsetAsync(s->st, 0, sizeof(PcgState), s->stream));
-    IFL_HIP(hipHostMalloc((void**)&s->st_host, sizeof(PcgState), hipHostMallocDefault));
-    memset(s->st_host, 0, sizeof(PcgState));
+    IFL_HIP(hipHostMalloc((void**)&s->st_host, 2 * sizeof(PcgState), hipHostMallocDefault));
+    memset(s->st_host, 0, 2 * sizeof(PcgState));
     s->stage_count = (size_t)(W + 2) * (H + 2);
     IFL_TRY(dalloc(s, &s->stage_buf, s->stage_count));
     long cap = (long)(W + 1) * (H + 1);

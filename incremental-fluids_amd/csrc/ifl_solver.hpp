@@ -81,7 +81,8 @@ struct Solver {
     double* partial = nullptr;            // per-block partial reductions
     int npartial = 0;
     PcgState* st = nullptr;
-    PcgState* st_host = nullptr;          // pinned mirror
+    PcgState* st_host = nullptr;          // pinned mirrors (two, by turns)
+    hipEvent_t ev_group[2] = {nullptr, nullptr};  // after a mirror's copy
     double* stage_buf = nullptr;          // row-major staging for layout conversion / upload
     size_t stage_count = 0;
 

@@ -256,7 +256,8 @@ IFL_DEV const const_u64* strip_masks(const StreamArgs& a, int j) {
 // (MODE 1) the loader forms r + q*(-alpha) (scaledAdd 7:870; at FLUID cells
 // only from level 6 on) and keeps only the result.
 template <int KIND, int MODE, int LV, int NG, typename T>
-IFL_DEV void loader_wave(const StreamArgs& a, char* ring, int k, int lane, long sbase, int nblk, int j) {
+IFL_DEV void loader_wave(const StreamArgs& a, char* ring, int k, int lane, long sbase, int nblk, int j,
+                         bool skip) {
     typedef SweepShape<KIND, MODE, NG, T> S;
     constexpr int R = S::R, NL = S::NLD;
     constexpr int kLoaders = loaders(KIND);
@@ -347,6 +348,7 @@ IFL_DEV void loader_wave(const StreamArgs& a, char* ring, int k, int lane, long 
     if (nmine > 0) issue(0, b0, w0);
     if (R > 1 && nmine > 1) issue(1, b1, w1);
     if (R > 2 && nmine > 2) issue(2, b2, w2);
+    if (skip) return;
     for (int i = 0; i < nmine; i += R) {
         if (!stage(i, b0, w0)) return;
         if (R > 1 && !stage(i + 1, b1, w1)) return;
@@ -804,10 +806,12 @@ template <int KIND, int MODE, int LV, int NG, typename T, bool TR>
 IFL_DEV void sweep_body(const StreamArgs& a, int j) {
     char* smem = sweep_smem;
     PcgState* st = a.st;
-    if (KIND != SW_PRECON && ((MODE >= 1 && st->done) || st->timeout)) return;
     // inside the PCG loop the backward sweep follows the convergence test
-    // (7:872-876): it does nothing once max|r| < tol (a.sigma holds tol)
-    if (KIND == SW_BWD && MODE == 1 && st->max_err < a.sigma) return;
+    // (7:872-876): it does nothing once max|r| < tol (a.sigma holds tol).
+    // The loaders test `skip` after their first loads have gone out, so the
+    // state's round trip and theirs overlap.
+    const bool skip = KIND != SW_PRECON &&
+                      ((MODE >= 1 && st->done) || st->timeout || (KIND == SW_BWD && MODE == 1 && st->max_err < a.sigma));
     double* ering = (double*)(smem + sizeof(RingHdr));
     char* ring = smem + sizeof(RingHdr) + kERing * sizeof(double);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -822,7 +826,11 @@ IFL_DEV void sweep_body(const StreamArgs& a, int j) {
     const double* ein = has_in ? a.edge + (long)(KIND == SW_BWD ? j + 1 : j) * W : nullptr;
     double* eout = has_out ? a.edge + (long)(KIND == SW_BWD ? j : j + 1) * W : nullptr;
 
-    if (wave == kWaveCompute)
+    if (loader_of_wave<KIND>(wave) >= 0)
+        loader_wave<KIND, MODE, LV, NG, T>(a, ring, loader_of_wave<KIND>(wave), lane, sbase, nblk, j, skip);
+    else if (skip)
+        return;
+    else if (wave == kWaveCompute)
         compute_wave<KIND, MODE, NG, T, TR>(a, ring, ering, j, lane);
     else if (wave == kWaveWriter)
         writer_wave<KIND, MODE, LV, NG, T, TR>(a, ring, j, lane, eout);
@@ -830,8 +838,6 @@ IFL_DEV void sweep_body(const StreamArgs& a, int j) {
         poller_wave<KIND>(a, ein, ering, lane);
     else if (KIND == SW_BWD && wave == kWaveDot)
         dot_wave<MODE, LV, NG, T>(a, ring, j, lane);
-    else if (loader_of_wave<KIND>(wave) >= 0)
-        loader_wave<KIND, MODE, LV, NG, T>(a, ring, loader_of_wave<KIND>(wave), lane, sbase, nblk, j);
 }
 
 // The sweep kernels that deal a launch's strips upstream first
