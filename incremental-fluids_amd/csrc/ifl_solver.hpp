@@ -58,7 +58,7 @@ struct Solver {
     Skew sk;
     size_t sk_count = 0;
     double *r = nullptr, *p = nullptr, *z = nullptr, *s = nullptr;
-    // levels 6-8, FP64 with tree-ordered dots: the PCG iterations after the
+    // levels 3 and 6-8, FP64 with tree-ordered dots: the PCG iterations after the
     // first form s = z + beta s inside the matrix-vector product, writing the
     // new s here and in s by turns (null: not used)
     double* s2 = nullptr;

@@ -151,14 +151,21 @@ __global__ __launch_bounds__(256) void matvec_kernel(VecArgs a, int check_done) 
     matvec_body<OUT_Q>(a, blockIdx.x, check_done);
 }
 
-// A1 and A2 in one pass, for vector operations masked to FLUID cells (levels
-// 6-8) in the FP64 form: scaledAdd(_p, _p, _s, alpha) 7:869 and
-// scaledAdd(_s, _z, _s, beta) 7:881 of the previous iteration, then
-// matrixVectorProduct(_z, _s) 7:868 and the block partial of its dot
-// product. Each product term takes its neighbour's new s as that update
-// forms it (z + s beta at a FLUID cell, s unchanged elsewhere), so the terms
-// are vec_update_kernel's and matvec_kernel's values; the new s goes to a
-// second array, since neighbouring workgroups still read the old one.
+// A1 and A2 in one pass, in the FP64 form with tree-ordered dots:
+// scaledAdd(_p, _p, _s, alpha) 7:869 and scaledAdd(_s, _z, _s, beta) 7:881 of
+// the previous iteration, then matrixVectorProduct(_z, _s) 7:868 and the block
+// partial of its dot product. Each product term takes its neighbour's new s
+// as that update forms it, so the terms are vec_update_kernel's and
+// matvec_kernel's values; the new s goes to a second array, since
+// neighbouring workgroups still read the old one.
+// VM (levels 6-8): vector operations touch FLUID cells only. Level 3 updates
+// every cell, and every cell is FLUID: one launch and one pass over s and p
+// fewer, 55.8 -> 51.9 us per iteration at 128^2 and 51.4 -> 48.6 at 96x80.
+// Levels 4-5 keep the two kernels: their update takes A s at non-FLUID cells,
+// which the fused form could only read from z, and the backward sweep's
+// writer, storing it there, set the sweep's pace (batch of 64 solvers of
+// level 4: 101 against 78 us per launch, for 47 against 50 us here).
+template <bool VM>
 IFL_DEV void matvec_update_body(const VecArgs& a, long blk, const double* __restrict__ so, double* __restrict__ sn) {
     __shared__ double red[4];
     PcgState* st = a.st;
@@ -179,13 +186,13 @@ IFL_DEV void matvec_update_body(const VecArgs& a, long blk, const double* __rest
         const long js = hs ? (l > 0 ? i - kStrip - 1 : sk.pos(x, y - 1)) : i;
         const long je = he ? i + kStrip : i;
         const long jn = hn ? (l < kStrip - 1 ? i + kStrip + 1 : sk.pos(x, y + 1)) : i;
-        const bool fl = a.flag[i] != 0, fw = a.flag[jw] != 0, fs = a.flag[js] != 0, fe = a.flag[je] != 0,
-                   fn = a.flag[jn] != 0;
+        auto on = [&](long c) { return !VM || a.flag[c] != 0; };
+        const bool fl = on(i), fw = on(jw), fs = on(js), fe = on(je), fn = on(jn);
         const double s0 = so[i], sw = so[jw], ss = so[js], se = so[je], snn = so[jn];
         const double z0 = a.z[i], zw = a.z[jw], zs = a.z[js], ze = a.z[je], zn = a.z[jn];
         const double ad = a.adiag[i], axw = a.apx[jw], ays = a.apy[js], ax = a.apx[i], ay = a.apy[i];
         const double p0 = a.p[i];
-        // the new s (z + s beta at a FLUID cell, s elsewhere)
+        // the new s (z + s beta where the update reaches, s elsewhere)
         const double b = fl ? z0 + s0 * beta : s0;
         const double bw = fw ? zw + sw * beta : sw;
         const double bs = fs ? zs + ss * beta : ss;
@@ -206,9 +213,10 @@ IFL_DEV void matvec_update_body(const VecArgs& a, long blk, const double* __rest
     __syncthreads();
     if (threadIdx.x == 0) a.partial[blk] = (red[0] + red[1]) + (red[2] + red[3]);
 }
+template <bool VM>
 __global__ __launch_bounds__(256) void matvec_update_kernel(VecArgs a, const double* __restrict__ so,
                                                             double* __restrict__ sn) {
-    matvec_update_body(a, blockIdx.x, so, sn);
+    matvec_update_body<VM>(a, blockIdx.x, so, sn);
 }
 
 // Fixed-order sum of `n` partials by one workgroup of 256 threads.
@@ -853,7 +861,7 @@ __global__ void defl_init_s_kernel(VecArgs a) {
 // already done.
 // iterations fuse the vector update into the product (matvec_update_kernel)
 static bool fused_update(const Solver* s, const VecArgs& a) {
-    return s->s2 && s->cfg.dot_order == IFL_DOT_TREE && a.vm && !a.defl;
+    return s->s2 && s->cfg.dot_order == IFL_DOT_TREE && !a.defl;
 }
 // the array holding s after iteration `it` (s and s2 by turns when fused)
 static double* s_after(Solver* s, int it) { return s->s2 && it > 0 && (it & 1) ? s->s2 : s->s; }
@@ -870,7 +878,10 @@ static int launch_iteration(Solver* s, int it, int limit) {
     }
     IFL_TRY(prof_begin(s, IFL_KERNEL_MATVEC, it));
     if (it > 0 && fuse) {
-        matvec_update_kernel<<<nbv, 256, 0, s->stream>>>(a, s_after(s, it - 1), s_after(s, it));
+        if (a.vm)
+            matvec_update_kernel<true><<<nbv, 256, 0, s->stream>>>(a, s_after(s, it - 1), s_after(s, it));
+        else
+            matvec_update_kernel<false><<<nbv, 256, 0, s->stream>>>(a, s_after(s, it - 1), s_after(s, it));
     } else {
         matvec_kernel<1><<<nbv, 256, 0, s->stream>>>(a, 1);
     }
@@ -1327,7 +1338,8 @@ struct BatchDev {
     int nvblk4 = 0;
     int nvblk_full = 0, nsblk_full = 0;
     bool compacted = false;
-    bool fused = false;  // the vector update folded into the product (every instance: levels 6-8 with s2)
+    bool fused = false;  // the vector update folded into the product (every instance: levels 3 and 6-8 with s2)
+    bool masked = false;  // vector operations masked to FLUID cells (levels 6-8)
     // profiling: events around the fused launches (matvec, forward and
     // backward sweep) of the current solve
     std::vector<hipEvent_t> ev_pool;
@@ -1458,16 +1470,17 @@ __global__ __launch_bounds__(256) void batch_matvec_kernel(const BatchInst* t, c
 }
 
 // matvec_update_body for every instance: the vector update of iteration
-// it - 1 and the product of iteration it in one pass (levels 6-8), one block
+// it - 1 and the product of iteration it in one pass, one block
 // of an instance per workgroup; s is read from the array iteration it - 1
 // left it in and the new s goes to the other. (Four blocks per workgroup, the
 // block reduction's LDS reused between them: 25.3 against 23.7 us per launch
 // on 16 FLIP instances at 256^2.)
+template <bool VM>
 __global__ __launch_bounds__(256) void batch_matvec_update_kernel(const BatchInst* t, const int2* map, int it) {
     const int2 m = map[blockIdx.x];
     const BatchInst& b = t[m.x];
     const VecArgs a = b.v;
-    matvec_update_body(a, m.y, batch_s_after(b, it - 1), batch_s_after(b, it));
+    matvec_update_body<VM>(a, m.y, batch_s_after(b, it - 1), batch_s_after(b, it));
 }
 
 __global__ __launch_bounds__(256) void batch_fin_alpha_kernel(const BatchInst* t) {
@@ -1650,8 +1663,9 @@ int batch_build(Solver* const* ss, int n, BatchDev* d) {
     d->fmap_h = fmap;
     d->bmap_h = bmap;
     // the vector update folds into the product when every instance can, as
-    // for one solver (fused_update: the second s, tree dots, masked vectors)
+    // for one solver (fused_update: the second s, tree dots)
     d->fused = true;
+    d->masked = inst[0].v.vm != 0;
     for (int i = 0; i < n; i++) d->fused = d->fused && fused_update(ss[i], inst[i].v);
     for (int i = 0; i < n; i++) inst[i].s2 = d->fused ? ss[i]->s2 : nullptr;
     IFL_TRY(upload(s, &d->inst, inst));
@@ -1710,7 +1724,10 @@ int batch_iteration(Solver* s, BatchDev* d, hipStream_t stream, int it, bool pro
     }
     if (prof) IFL_TRY(batch_time(s, d, stream, IFL_KERNEL_MATVEC, true));
     if (fuse)
-        batch_matvec_update_kernel<<<d->nvblk, 256, 0, stream>>>(d->inst, d->vmap, it);
+        if (d->masked)
+            batch_matvec_update_kernel<true><<<d->nvblk, 256, 0, stream>>>(d->inst, d->vmap, it);
+        else
+            batch_matvec_update_kernel<false><<<d->nvblk, 256, 0, stream>>>(d->inst, d->vmap, it);
     else
         batch_matvec_kernel<<<d->nvblk4, 256, 0, stream>>>(d->inst, d->vmap4);
     IFL_LAUNCH_CHECK();
