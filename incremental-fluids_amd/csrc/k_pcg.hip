@@ -1183,31 +1183,45 @@ int k_project(Solver* s, int limit, ifl_solve_stats* stats) {
         fin_sigma_kernel<<<1, 256, 0, s->stream>>>(a, s->sk.nstrips, seq, 1, s->cfg.tol, limit);  // 7:858-864
         IFL_LAUNCH_CHECK();
     }
-    // Iterations go out in groups, one group ahead of the state the host waits
-    // for, so the device has work while the host reads; past the exit a launch
-    // returns at once. Groups of 8 (4 at first): a solve that ends runs 4 + 8
-    // such iterations on average (~10 us each), where groups doubling from 4
-    // to 64 ran 50 for 74 that worked (128^2) and waited on every read; a
-    // group's state copy is under 1 % of it at 96x80.
+    // Iterations go out in groups of 4, after 16 of 8; past the exit a launch
+    // returns at once (~10 us for an iteration's). The host waits for the
+    // entry's state and the first group's, since many solves end there, and
+    // then stays one group ahead of the state it waits for, so the device has
+    // work while the host reads. A solve of 74 iterations (128^2) launches 92;
+    // groups doubling from 4 to 64 launched 124 and left the device idle at
+    // every read.
     int launched = 0, group = 0;
     PcgState h;
-    auto launch_group = [&]() -> int {
-        const int nb = std::min(launched < 8 ? 4 : 8, limit - launched);
-        for (int k = 0; k < nb; k++) IFL_TRY(launch_iteration(s, launched + k, limit));
-        launched += std::max(nb, 0);
+    auto post = [&]() -> int {  // the state after what has been launched
         IFL_HIP(hipMemcpyAsync(&s->st_host[group & 1], s->st, sizeof(PcgState), hipMemcpyDeviceToHost, s->stream));
         IFL_HIP(hipEventRecord(s->ev_group[group & 1], s->stream));
         group++;
         return IFL_OK;
     };
-    IFL_TRY(launch_group());
-    while (true) {
-        const bool last = launched >= limit;
-        if (!last) IFL_TRY(launch_group());
-        const int seen = (last ? group - 1 : group - 2) & 1;
-        IFL_HIP(hipEventSynchronize(s->ev_group[seen]));
-        h = s->st_host[seen];
-        if (h.done || h.timeout || last) break;
+    auto launch_group = [&]() -> int {
+        const int nb = std::min(launched < 16 ? 4 : 8, limit - launched);
+        for (int k = 0; k < nb; k++) IFL_TRY(launch_iteration(s, launched + k, limit));
+        launched += nb;
+        return post();
+    };
+    bool ahead = false;  // a group beyond the state waited for is in flight
+    auto wait = [&]() -> int {
+        const int g = ahead ? group - 2 : group - 1;
+        if (ahead)
+            IFL_HIP(hipEventSynchronize(s->ev_group[g & 1]));
+        else
+            IFL_HIP(hipStreamSynchronize(s->stream));  // returns ~10 us sooner than the event's wait
+        h = s->st_host[g & 1];
+        return IFL_OK;
+    };
+    IFL_HIP(hipMemcpyAsync(&s->st_host[1], s->st, sizeof(PcgState), hipMemcpyDeviceToHost, s->stream));
+    IFL_HIP(hipStreamSynchronize(s->stream));
+    h = s->st_host[1];
+    while (!h.done && !h.timeout && (ahead || launched < limit)) {
+        if (!ahead) IFL_TRY(launch_group());
+        ahead = launched > 4 && launched < limit;
+        if (ahead) IFL_TRY(launch_group());
+        IFL_TRY(wait());
     }
     if (h.timeout) {
         s->err = "PCG sweep hand-off timed out";

@@ -1,4 +1,4 @@
-// The streamed MIC(0) sweeps: ring layout, the six waves' roles and the
+// The streamed MIC(0) sweeps: ring layout, the eight waves' roles and the
 // per-strip body (see k_pcg.hip for the PCG around them). Included by
 // k_pcg.hip, whose kernels deal strips grouped by XCD, and by k_sweep_up.hip,
 // whose kernels deal them upstream first.
@@ -32,7 +32,8 @@ IFL_DEV uint64_t as_bits(double v) { return (uint64_t)__double_as_longlong(v); }
 //           always run and no strip needs the others resident.
 // Order 1 is used when the strips outnumber the CUs or when another solver
 // is stepping on the device at the same time; alone, order 0 measured
-// faster at 2048^2 (forward / backward 384 / 356 us, against 388 / 400 us).
+// faster at 2048^2 (forward / backward 384 / 356 us,
+// against 388 / 400 us, measured with six waves per strip).
 IFL_DEV int strip_of_block(int b, int n, bool reverse, int order) {
     if (order) return b < n ? (reverse ? n - 1 - b : b) : -1;
     int per = (n + 7) >> 3;
@@ -122,11 +123,10 @@ struct StreamArgs {
     double tau, sigma;      // the factor build's tau and sigma (7:743-744); the PCG
                             // loop's backward sweep: sigma = the convergence tolerance
     int strip0, nlaunch;    // the strips of this launch
-    int pad;                // unused: keeps the fields below where the sweeps were
-                            // measured fastest (without it 388 / 363 us per forward /
-                            // backward sweep at 2048^2, with it 384 / 357 us, the
-                            // same box and code: the layout moves the kernels'
-                            // argument loads and their schedule)
+    int pad;                // unused: keeps the fields below where the six-wave form of
+                            // these sweeps was fastest (384 / 357 us per forward / backward
+                            // sweep at 2048^2, 388 / 363 without it: the layout moves the
+                            // kernels' argument loads); not measured again since
     int nb;                 // ring depth in blocks
     int slot_bytes;         // bytes of one ring slot
     long long* trace;       // diagnostics: kTraceStamps stamps per strip and block, or null
@@ -228,7 +228,7 @@ struct SweepShape {
     static constexpr int NLD = lo(NG);  // 1 KB loads per block
     static constexpr int OUT = ro(NS);  // output region
     static constexpr int SLOT = OUT + 512 * (KIND == SW_PRECON ? 8 : (int)sizeof(T));
-    static constexpr int R = NLD <= 16 ? 3 : 2;  // blocks in flight per loader, 4 VGPRs per load
+    static constexpr int R = NLD < 16 ? 3 : 2;  // blocks in flight per loader, 4 VGPRs per load (3 of 16 spill)
     // arrays wave 0 reads in precision T, and where they are in the slot
     static constexpr int NT = KIND == SW_BWD ? 4 : 3;
     static constexpr int tarr(int i) { return KIND == SW_FWD ? i + 1 : i; }
