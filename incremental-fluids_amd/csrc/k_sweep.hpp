@@ -468,8 +468,8 @@ IFL_DEV void compute_wave(const StreamArgs& a, char* ring, const double* ering, 
     // would wait for the loads): X[i][p] holds steps 2p and 2p+1 of the i-th
     // T array (one ds_read2st64), Q[p] those of the updated residual (forward
     // sweep), E[p] the two edge values of those steps, M0/M1 the eight lane
-    // masks in column order (scalar loads). The reads of block b+1 go out at
-    // the start of block b.
+    // masks in column order (scalar loads). The reads of block b+1 go out
+    // between the steps of block b.
     typedef uint64_t vec4u __attribute__((ext_vector_type(4)));
     typedef const __attribute__((address_space(4))) vec4u const_u64x4;
     constexpr int NP = kBlk / 2;
