@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "ifl_solver.hpp"
+#include "k_groups.hpp"
 #include "k_sweep.hpp"
 
 namespace ifl {
@@ -1183,46 +1184,36 @@ int k_project(Solver* s, int limit, ifl_solve_stats* stats) {
         fin_sigma_kernel<<<1, 256, 0, s->stream>>>(a, s->sk.nstrips, seq, 1, s->cfg.tol, limit);  // 7:858-864
         IFL_LAUNCH_CHECK();
     }
-    // Iterations go out in groups of 4, after 16 of 8; past the exit a launch
-    // returns at once (~10 us for an iteration's). The host waits for the
-    // entry's state and the first group's, since many solves end there, and
-    // then stays one group ahead of the state it waits for, so the device has
-    // work while the host reads. A solve of 74 iterations (128^2) launches 92;
-    // groups doubling from 4 to 64 launched 124 and left the device idle at
-    // every read.
-    int launched = 0, group = 0;
-    PcgState h;
-    auto post = [&]() -> int {  // the state after what has been launched
-        IFL_HIP(hipMemcpyAsync(&s->st_host[group & 1], s->st, sizeof(PcgState), hipMemcpyDeviceToHost, s->stream));
-        IFL_HIP(hipEventRecord(s->ev_group[group & 1], s->stream));
-        group++;
-        return IFL_OK;
-    };
-    auto launch_group = [&]() -> int {
-        const int nb = std::min(launched < 16 ? 4 : 8, limit - launched);
-        for (int k = 0; k < nb; k++) IFL_TRY(launch_iteration(s, launched + k, limit));
-        launched += nb;
-        return post();
-    };
-    bool ahead = false;  // a group beyond the state waited for is in flight
-    auto wait = [&]() -> int {
-        const int g = ahead ? group - 2 : group - 1;
-        if (ahead)
-            IFL_HIP(hipEventSynchronize(s->ev_group[g & 1]));
-        else
-            IFL_HIP(hipStreamSynchronize(s->stream));  // returns ~10 us sooner than the event's wait
-        h = s->st_host[g & 1];
-        return IFL_OK;
-    };
-    IFL_HIP(hipMemcpyAsync(&s->st_host[1], s->st, sizeof(PcgState), hipMemcpyDeviceToHost, s->stream));
-    IFL_HIP(hipStreamSynchronize(s->stream));
-    h = s->st_host[1];
-    while (!h.done && !h.timeout && (ahead || launched < limit)) {
-        if (!ahead) IFL_TRY(launch_group());
-        ahead = launched > 4 && launched < limit;
-        if (ahead) IFL_TRY(launch_group());
-        IFL_TRY(wait());
-    }
+    // the iterations (run_groups): their launches and the state's two pinned mirrors
+    struct Queue {
+        Solver* s;
+        int limit;
+        int launch(int it) { return launch_iteration(s, it, limit); }
+        int copy(int m) {
+            IFL_HIP(hipMemcpyAsync(&s->st_host[m], s->st, sizeof(PcgState), hipMemcpyDeviceToHost, s->stream));
+            return IFL_OK;
+        }
+        int post(int m) {
+            IFL_TRY(copy(m));
+            IFL_HIP(hipEventRecord(s->ev_group[m], s->stream));
+            return IFL_OK;
+        }
+        int wait(int m, bool all) {
+            if (all)
+                IFL_HIP(hipStreamSynchronize(s->stream));  // returns ~10 us sooner than the event's wait
+            else
+                IFL_HIP(hipEventSynchronize(s->ev_group[m]));
+            return IFL_OK;
+        }
+        bool over(int m) { return s->st_host[m].done || s->st_host[m].timeout; }
+        bool seen_over(int m) { return ((const volatile PcgState*)s->st_host)[m].done != 0; }
+    } queue{s, limit};
+    int last = 1;
+    IFL_TRY(queue.copy(last));
+    IFL_TRY(queue.wait(last, true));
+    if (!queue.over(last) && limit > 0)
+        IFL_TRY(run_groups(queue, limit, short_iterations(s->W, s->sk.nstrips), &last));
+    const PcgState h = s->st_host[last];
     if (h.timeout) {
         s->err = "PCG sweep hand-off timed out";
         (void)edge_reset(s);
