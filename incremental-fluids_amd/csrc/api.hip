@@ -337,11 +337,14 @@ int init_solver(Solver* s) {
                        &s->cx, &s->cy, &s->yv, &s->qv};
     for (double** a : arrs) IFL_TRY(dalloc(s, a, n));
     IFL_TRY(balloc(s, &s->dflag, n));
-    // the fused vector update of the PCG iterations (levels 3 and 6-8, FP64);
-    // IFL_NO_FUSED_UPDATE=1 in the environment at creation keeps the
-    // separate update kernel (diagnostics: the two give identical iterates)
+    // the fused vector update of the PCG iterations (levels 3 and 6-8, FP64,
+    // tree-ordered dots); IFL_NO_FUSED_UPDATE=1 in the environment at creation
+    // keeps the separate update kernel (diagnostics: the two give identical
+    // iterates)
     const char* nofuse = getenv("IFL_NO_FUSED_UPDATE");
-    if ((lv == 3 || lv >= 6) && s->cfg.precision == IFL_PREC_FP64 && !(nofuse && nofuse[0] == '1')) IFL_TRY(dalloc(s, &s->s2, n));
+    if ((lv == 3 || lv >= 6) && s->cfg.precision == IFL_PREC_FP64 && s->cfg.dot_order == IFL_DOT_TREE &&
+        !(nofuse && nofuse[0] == '1'))
+        IFL_TRY(dalloc(s, &s->s2, n));
     if (s->cfg.precision != IFL_PREC_FP64) {
         float** sarrs[] = {&s->cx32, &s->cy32, &s->pc32, &s->y32, &s->e32, &s->r32, &s->s32,
                            &s->z32, &s->q32, &s->ad32, &s->apx32, &s->apy32};
