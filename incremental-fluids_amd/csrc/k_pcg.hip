@@ -1343,7 +1343,7 @@ struct BatchDev {
     int nvblk4 = 0;
     int nvblk_full = 0, nsblk_full = 0;
     bool compacted = false;
-    bool fused = false;  // the vector update folded into the product (every instance: levels 3 and 6-8 with s2)
+    bool fused = false;  // the vector update folded into the product (every instance has s2: levels 6-8, and 3 up to kFoldCells)
     bool masked = false;  // vector operations masked to FLUID cells (levels 6-8)
     // profiling: events around the fused launches (matvec, forward and
     // backward sweep) of the current solve
@@ -1373,6 +1373,9 @@ namespace {
 // matrix-vector product: an instance's arguments are loaded once for all of
 // them (each block's partial is the single-solver kernel's)
 constexpr int kVecBlocks = 4;
+
+// cells of the largest level 3 batch that folds the vector update into the product
+constexpr long kFoldCells = 2000000;
 
 // vec_update_body (mode 0) over kVecBlocks blocks at once, every load of the
 // workgroup's cells issued before the first store; each cell's values are
@@ -1671,7 +1674,19 @@ int batch_build(Solver* const* ss, int n, BatchDev* d) {
     // for one solver (fused_update: the second s, tree dots)
     d->fused = true;
     d->masked = inst[0].v.vm != 0;
-    for (int i = 0; i < n; i++) d->fused = d->fused && fused_update(ss[i], inst[i].v);
+    long cells = 0;
+    for (int i = 0; i < n; i++) {
+        d->fused = d->fused && fused_update(ss[i], inst[i].v);
+        cells += (long)ss[i]->W * ss[i]->H;
+    }
+    // At level 3 only in batches of up to 2M cells: above, the one-block fused
+    // product costs more than the launch it saves. Step folded / with the two
+    // kernels: 4 instances of 96x80 2.9 / 3.1 ms, 32 of mixed sizes (1.98M
+    // cells) 59.5 / 59.8, 8 of 512x512 (2.1M) 64.1 / 63.3, 256 of 128x128 (4.2M)
+    // 23.5 / 22.8, 32 of 512x512 (8.4M) 123.8 / 121.1. Levels 6-8, where FLUID
+    // masks leave cells out, gain or tie at most sizes (level 7: 3.6 / 4.0,
+    // 60.4 / 61.9, 69.0 / 68.4, 28.1 / 27.0, 139.1 / 139.1).
+    if (!d->masked && cells > kFoldCells) d->fused = false;
     for (int i = 0; i < n; i++) inst[i].s2 = d->fused ? ss[i]->s2 : nullptr;
     IFL_TRY(upload(s, &d->inst, inst));
     IFL_TRY(upload(s, &d->fwd, fwd));
