@@ -503,7 +503,6 @@ static int launch_stream_k(Solver* s, StreamArgs a) {
         attr_set.store(true, std::memory_order_release);
     }
     a.nlaunch = s->sk.nstrips;
-    a.strip0 = 0;
     // the traced sweeps (diagnostics) always run alone
     if (!TR && (a.nlaunch > s->num_cus || (s->busy && s->busy->load(std::memory_order_relaxed) > 1)))
         return launch_sweep_up<KIND, MODE, LV, NG, T>(s, a, shmem);
@@ -605,8 +604,9 @@ int k_build_precon(Solver* s) {
 }
 
 // Diagnostics: one sweep of `kind` on the current state, time-stamped per
-// block (100 MHz clock): wave 0 starts the block, its operands for the
-// second half are ready, the writer has drained it.
+// block (100 MHz clock): wave 0 begins the block, the next block's operands
+// and edges are in LDS, wave 0 has computed it, the writer has drained it
+// (stamps 0, 1, 4 and 5).
 int k_trace_sweep(Solver* s, int kind, long long* dev_trace) {
     if (kind == SW_PRECON) return launch_precon(s, dev_trace);
     if (kind == SW_FWD) return launch_fwd<0>(s, dev_trace);
@@ -1493,11 +1493,6 @@ __global__ __launch_bounds__(256) void batch_matvec_update_kernel(const BatchIns
 
 __global__ __launch_bounds__(256) void batch_fin_alpha_kernel(const BatchInst* t) {
     fin_alpha_body(t[blockIdx.x].v, t[blockIdx.x].nbv, 0);
-}
-
-__global__ void batch_fin_check_kernel(const BatchInst* t, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) fin_check_body(t[i].v.st, t[i].tol);
 }
 
 __global__ __launch_bounds__(256) void batch_fin_sigma_kernel(const BatchInst* t) {

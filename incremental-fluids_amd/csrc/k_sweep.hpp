@@ -31,9 +31,9 @@ IFL_DEV uint64_t as_bits(double v) { return (uint64_t)__double_as_longlong(v); }
 //           n - 1 - b of a backward one), so the lowest unfinished strip can
 //           always run and no strip needs the others resident.
 // Order 1 is used when the strips outnumber the CUs or when another solver
-// is stepping on the device at the same time; alone, order 0 measured
-// faster at 2048^2 (forward / backward 384 / 356 us,
-// against 388 / 400 us, measured with six waves per strip).
+// is stepping on the device at the same time; alone, order 0 is the same or
+// faster (us per PCG iteration, order 0 / 1: 2048^2 747.7 / 747.3, 1000x777
+// 282.4 / 283.1, 512^2 163.0 / 164.1, 128^2 50.3 / 50.7).
 IFL_DEV int strip_of_block(int b, int n, bool reverse, int order) {
     if (order) return b < n ? (reverse ? n - 1 - b : b) : -1;
     int per = (n + 7) >> 3;
@@ -122,24 +122,18 @@ struct StreamArgs {
     int* timeout;
     double tau, sigma;      // the factor build's tau and sigma (7:743-744); the PCG
                             // loop's backward sweep: sigma = the convergence tolerance
-    int strip0, nlaunch;    // the strips of this launch
-    int pad;                // unused: keeps the fields below where the six-wave form of
-                            // these sweeps was fastest (384 / 357 us per forward / backward
-                            // sweep at 2048^2, 388 / 363 without it: the layout moves the
-                            // kernels' argument loads); not measured again since
+    int nlaunch;            // the strips of this launch
+    int pad[2];             // unused: puts the fields below where the kernels' argument loads
+                            // schedule best (us per PCG iteration with / without: 2048^2
+                            // 747.1 / 748.0, 1000x777 281.1 / 281.7, 512^2 mixed 165.0 / 165.9)
     int nb;                 // ring depth in blocks
     int slot_bytes;         // bytes of one ring slot
     long long* trace;       // diagnostics: kTraceStamps stamps per strip and block, or null
 };
 
-// s_waitcnt with only vmcnt constrained (gfx9 encoding: vmcnt in bits 3:0
-// and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima).
-#define IFL_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (0x7 << 4) | (0xF << 8) | (((n) >> 4) << 14))
-
-// LDS counters are read and written through inline asm: the compiler would
-// otherwise wait for every in-flight LDS-DMA load (vmcnt(0)) before any LDS
-// instruction in the loaders, and it must not move ring accesses across a
-// counter access in any wave ("memory" clobber).
+// LDS counters are read and written through inline asm: a read waits for
+// itself alone, and the compiler must not move ring accesses across a counter
+// access in any wave ("memory" clobber).
 // The header sits at the start of the workgroup's dynamic LDS; its fields are
 // addressed by their LDS byte offsets (a generic pointer would cost a null
 // check at every use).
