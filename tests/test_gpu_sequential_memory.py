@@ -2,6 +2,8 @@
 only the fused vector update of tree-ordered dots uses one (levels 3 and 6-8).
 Its device memory is a solver's without the fused update, one array of
 doubles over the skewed layout less than with it."""
+import ctypes
+
 import pytest
 
 import oracle_lib as ol
@@ -12,17 +14,23 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("level", [3, 7])
 def test_no_second_direction_array(level, monkeypatch):
-    torch = pytest.importorskip("torch")
     import ifl_fluids as F
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        # of the runtime that the library is linked to
+        assert F.lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
     sc = ol.REF_SCENES[level]
     w, h = 2000, 1900
     make_product(level, 16, 16, sc["params"], []).close()  # the library's own one-time memory
 
     def held(order, fused):
         monkeypatch.setenv("IFL_NO_FUSED_UPDATE", "0" if fused else "1")
-        before = torch.cuda.mem_get_info()[0]
+        before = free_bytes()
         s = make_product(level, w, h, sc["params"], [], dot_order=order)
-        n = before - torch.cuda.mem_get_info()[0]
+        n = before - free_bytes()
         s.close()
         return n
 
@@ -30,4 +38,4 @@ def test_no_second_direction_array(level, monkeypatch):
     tree, plain, seq = held(F.DOT_TREE, True), held(F.DOT_TREE, False), held(F.DOT_SEQUENTIAL, True)
     print(f"level {level} {w}x{h}: tree {tree}, not fused {plain}, sequential {seq}, one array {array}", flush=True)
     assert tree - plain >= array // 2
-    assert seq == plain
+    assert abs(seq - plain) < array // 2
