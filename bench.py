@@ -36,7 +36,7 @@ KERNEL_BYTES_PER_CELL = {
 # the same for solver 4 (the batched form): its backward sweep also reads
 # the reference's _z at non-FLUID cells (A s, kept in q) for the unmasked dot
 BATCH_BYTES_PER_CELL = dict(KERNEL_BYTES_PER_CELL, sweep_bwd=56.0)
-# levels 6-8 in the FP64 form: the iterations after the first form the vector
+# levels 3 and 6-8 in the FP64 form: the iterations after the first form the vector
 # update inside the product (adiag, aplusx, aplusy, old s, z, p read; p, new
 # s, q written; the FLUID flags): timed as the product
 FUSED_MATVEC_BYTES_PER_CELL = 73.0
@@ -47,9 +47,9 @@ def kernel_bytes_per_cell(name, form):
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 # The order-preserving floor of a MIC(0) sweep: cell (x, y) needs (x-1, y) and
 # (x, y-1), so any schedule that keeps each cell's operations takes W + H - 1
-# dependent steps, each at least the recurrence's dependency chain (44 clocks,
+# dependent steps, each at least the recurrence's dependency chain (37 clocks,
 # measured in a one-wave loop of the compute step) at the 2.4 GHz engine clock.
-SWEEP_CHAIN_CLOCKS = 44
+SWEEP_CHAIN_CLOCKS = 37
 ENGINE_GHZ = 2.4
 
 

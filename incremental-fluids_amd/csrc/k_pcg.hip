@@ -162,10 +162,11 @@ __global__ __launch_bounds__(256) void matvec_kernel(VecArgs a, int check_done) 
 // VM (levels 6-8): vector operations touch FLUID cells only. Level 3 updates
 // every cell, and every cell is FLUID: one launch and one pass over s and p
 // fewer, 55.8 -> 51.9 us per iteration at 128^2 and 51.4 -> 48.6 at 96x80.
-// Levels 4-5 keep the two kernels: their update takes A s at non-FLUID cells,
-// which the fused form could only read from z, and the backward sweep's
-// writer, storing it there, set the sweep's pace (batch of 64 solvers of
-// level 4: 101 against 78 us per launch, for 47 against 50 us here).
+// Levels 4-5 keep the two kernels: their update takes A s at non-FLUID cells.
+// The backward sweep's writer merging it into z for the fused form set the
+// sweep's pace (batch of 64 solvers of level 4: 101 against 78 us per launch,
+// for 47 against 50 us here); reading the old q instead, which would take a
+// second q by turns as s has, was not built.
 template <bool VM>
 IFL_DEV void matvec_update_body(const VecArgs& a, long blk, const double* __restrict__ so, double* __restrict__ sn) {
     __shared__ double red[4];

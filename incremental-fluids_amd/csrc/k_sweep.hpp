@@ -241,9 +241,10 @@ IFL_DEV const const_u64* strip_masks(const StreamArgs& a, int j) {
 // CU streams 66 GB/s from HBM and 100 from the Infinity Cache with them, 59
 // and 56 with non-temporal ones, and what a sweep stores is read by the next
 // kernel (per PCG iteration: solver 7 at 2048^2 761 -> 747 us, at 1000x777
-// 317 -> 282, at 512^2 171 -> 163; the batch's launches 1-4 % faster). Up to
-// R blocks are in
-// flight in its registers (global_load_dwordx4: lane i holds bytes
+// 317 -> 282, at 512^2 171 -> 163; the batch's launches 1-4 % faster), though
+// at 2048^2 the product then finds less in the Infinity Cache (62 -> 67 us of
+// those). Up to R blocks are in flight in its registers
+// (global_load_dwordx4: lane i holds bytes
 // [16 i, 16 i + 16) of each 1 KB run of an array's block), so the prefetch
 // depth does not depend on free LDS slots; a block is written into its slot
 // once the slot is free. In the forward sweep with the residual update
